@@ -9,13 +9,9 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "knx_common.hpp"
+#include "knx_xgemm.hpp"
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-
-// the pipelined implicit-GEMM kernel (knx_sgemm.hip): returns 1 without launching when the shape does not qualify
-int knx_conv_k32(const knx_conv_geom* g, const float* x, const float* wt, const float* bias, int act, float alpha,
-                 const float* R, float* y, hipStream_t s, const char* name);
 
 namespace {
 
@@ -458,7 +454,15 @@ int conv_entry(const knx_conv_geom* g, const float* x, const float* w, const flo
         if (rc != 1) return rc;
     }
     if (TB) {
-        const int rc = knx_conv_k32(g, x, w, bias, act, alpha, R, y, s, name);
+        // KNX_CONV_TILE forces a tile of the bf16 kernel (tests, tuning)
+        static const struct { const char* name; int tile; } TILES[] = {
+            {"256x256", KNX_X256x128}, {"256x128", KNX_X256x128}, {"128x128", KNX_X128x128}, {"128x128w8", KNX_X128x128},
+            {"64x128", KNX_X64x64}, {"256x64", KNX_X256x64}, {"128x64", KNX_X128x64}};
+        const char* force = getenv("KNX_CONV_TILE");
+        int tile = 0;
+        for (const auto& t : TILES)
+            if (force != nullptr && strcmp(force, t.name) == 0) tile = t.tile;
+        const int rc = knx_xconv(g, x, w, bias, act, alpha, R, y, tile, s, name);
         if (rc != 1) return rc;
     }
     ConvArgs p{};
