@@ -4,18 +4,18 @@
 // the loop body of kernix_attention_run (reference include/kernix_model.h:1021-1046).  The Q/K/V/O projections
 // are ordinary Linear GEMMs run by the host (knx_hip_sgemm_ep).
 //
-// Paths: for dk = dv ∈ {32, 64, 128} and S ≤ 256 (S ≤ 128 at 128) one fused kernel keeps each head's K and V in
-// LDS and the scores in registers, so nothing but Q, K, V and the context touches HBM.  Otherwise one batched NT
-// MFMA GEMM writes all B·H score matrices (alpha = scale and the causal mask fused in its epilogue), the wavefront
-// softmax normalizes each row in place, and one batched GEMM multiplies by V and writes the context directly in the
-// (B·Rq) × (H·dv) layout the output projection reads; given scratch for Vᵀ, V is transposed once so that both
-// products have K-contiguous operands and run on the pipelined kernel.
+// Paths: dk = dv ≤ 128 runs as one kernel over tiles of 32 keys on the bf16 matrix cores (knx_flash.hip), or, for d = 32, 64
+// or 128 and S ≤ 64, as one kernel that keeps each head's K and V in LDS and the scores in registers, so nothing but Q, K, V and
+// the context touches HBM.  Otherwise, and where the heads are too few to fill the chip, one batched NT GEMM writes all
+// B·H score matrices (alpha = scale and the causal mask fused in its epilogue), the wavefront softmax normalizes each row
+// in place, and one batched GEMM multiplies by V and writes the context directly in the (B·Rq) × (H·dv) layout the output
+// projection reads; given scratch for Vᵀ, V is transposed once so that both products have K-contiguous operands.
 #include <stdlib.h>
 #include <string.h>
 
 #include <utility>
 
-#include "knx_pipe.hpp"
+#include "knx_flash.hpp"
 
 int knx_sgemm_batched(int M, int N, int K, const float* A, int lda, long long sAb, long long sAh, const float* B, int ldb,
                       long long sBb, long long sBh, bool transB, float* C, int ldc, long long sCb, long long sCh, int nb,
@@ -55,7 +55,7 @@ __device__ __forceinline__ void unrolled(F&& f, std::integer_sequence<int, T...>
 // 16 zero bytes: the source of the staged chunks of keys beyond S
 __device__ __attribute__((aligned(16))) float knx_attn_zero[4];
 
-// Fused attention for sequences of at most 32·NS keys, dk = dv = D ∈ {32, 64, 128}.  One block per (b·h, 128
+// Fused attention for sequences of at most 32·NS keys, dk = dv = D.  One block per (b·h, 128
 // queries), each wave owns 32 queries.  K_h and V_h of the whole sequence (zero beyond S) are staged in LDS by
 // LDS-DMA (global_load_lds, 16 bytes per lane), both row-major in 16-byte chunks with a per-row chunk swizzle, one
 // 32-key tile after another: the K tiles first, then the V tiles.  The wave computes Sᵀ = K_h·Q_hᵀ on 32×32×2 fp32
@@ -245,9 +245,8 @@ int launch_fused_d(const AttnArgs& a, hipStream_t s, const char* name)
 template <int NS, int D>
 int launch_fused(const AttnArgs& a, hipStream_t s, const char* name)
 {
-    // three 32-key tiles in flight up front, one more per consumed K tile: with all of K and V requested at once by
-    // every workgroup (64 KB each at S = 128, d = 64) a workgroup's first tile arrives anywhere in the 32 MB stream
-    // (B 64, H 8, S 128, d 64: 26.5 µs at depth 3, 26.7 at 2 and 4, 27.3 at 6, 27.8 with everything up front)
+    // three 32-key tiles in flight up front, one more per consumed K tile, so that a workgroup's first tile does not
+    // arrive anywhere in the stream of all workgroups' loads
     const char* dep = getenv("KNX_ATTN_DEPTH");  // tuning and tests: 2, 4, 6, or "all"
     if (dep != nullptr && strcmp(dep, "all") == 0) return launch_fused_d<NS, D, 2 * NS>(a, s, name);
     const int d = dep != nullptr ? atoi(dep) : 3;
@@ -257,36 +256,47 @@ int launch_fused(const AttnArgs& a, hipStream_t s, const char* name)
     return launch_fused_d<NS, D, 3>(a, s, name);
 }
 
-// the fused kernel when dk = dv ∈ {32, 64, 128}, S fits its LDS tiles and every row is 16-byte aligned; 1 = not eligible
+// what a caller may run without scratch for the scores: dk = dv ∈ {32, 64, 128}, S ≤ 256 (128), 16-byte aligned rows
+bool no_scratch(const AttnArgs& a)
+{
+    const bool small = a.S <= (a.dk == 128 ? 128 : 256) && (a.dk == 32 || a.dk == 64 || a.dk == 128);
+    return a.dk == a.dv && small && (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)a.V | (uintptr_t)a.ctx) & 15) == 0 &&
+           ((a.ldq | a.ldk | a.ldv) & 3) == 0 && (long long)a.B * a.H <= 65535;
+}
+
+// Whether the tiled kernel is the faster: a tile of 32 keys takes a workgroup 1.0, 1.6, 2.8 or 3.2 µs at d up to 32, 64, 96
+// and 128 (64: 2.6 with two workgroups on a CU); the GEMMs and the softmax 22 µs of launches, 16 bytes of traffic per
+// score and the products at 100 TFLOP/s.  Both measured: B 4, H 12, S 1000, d 64 85 against 203 µs; 15, 4, 351, 16: 19 / 59;
+// 1, 2, 2000, 128 (32 workgroups): 190 / 78.
+bool tiled_faster(const AttnArgs& a)
+{
+    const double groups = (double)a.B * a.H * ((a.Rq + 127) / 128), cus = knx::num_cus();
+    const double tile = a.dk <= 32 ? 1.0 : a.dk <= 64 ? (groups > cus ? 2.6 : 1.6) : a.dk <= 96 ? 2.8 : 3.2;
+    const double slots = a.dk <= 64 && groups > cus ? 2 * cus : cus;
+    double tiles = (a.S + 31) / 32;
+    if (a.causal && groups > slots) tiles = 0.5 * tiles + 2;
+    const double rounds = groups <= slots ? 1.0 : groups / slots;
+    const double pairs = (double)a.B * a.H * a.Rq * a.S;
+    return 8 + tiles * tile * rounds < 22 + pairs * 16 / 5e6 + 4.0 * pairs * a.dk / 1e8;
+}
+
+// the whole core as one kernel; 1 = not eligible
 int try_fused(const AttnArgs& a, hipStream_t s, const char* name)
 {
-    const char* force = getenv("KNX_ATTN_KERNEL");
+    const char* force = getenv("KNX_ATTN_KERNEL");  // "unfused", "flash" (tests)
     if (force != nullptr && strcmp(force, "unfused") == 0) return 1;
-    if (a.dk != a.dv || (((uintptr_t)a.Q | (uintptr_t)a.K | (uintptr_t)a.V | (uintptr_t)a.ctx) & 15) != 0 ||
-        ((a.ldq | a.ldk | a.ldv) & 3) != 0)
-        return 1;
-    if ((long long)a.B * a.H > 65535) return 1;  // grid.y
-    const int ns = a.S <= 32 ? 1 : a.S <= 64 ? 2 : a.S <= 128 ? 4 : a.S <= 256 ? 8 : 0;
-    if (ns == 0 || (a.dk == 128 && ns == 8)) return 1;
-#define KNX_FUSED_NS(D)                                         \
-    switch (ns) {                                              \
-    case 1: return launch_fused<1, D>(a, s, name);             \
-    case 2: return launch_fused<2, D>(a, s, name);             \
-    case 4: return launch_fused<4, D>(a, s, name);             \
-    default: return launch_fused<8, D>(a, s, name);            \
+    const bool flash = force != nullptr && strcmp(force, "flash") == 0;
+    // S ≤ 64: the whole head's loads go out at once here (59 × 2 heads of 15 keys, d 32: 4.9 µs, 6.1 on the tiled kernel; 40 × 8
+    // heads of 40 keys, d 128: 23.1 / 26.9); from there on tiles are the faster (30 × 12, 100 keys, d 64: 25.2 / 19.6)
+    if (!flash && a.S <= 64 && no_scratch(a)) {
+        const bool one = a.S <= 32;
+        if (a.dk == 32) return one ? launch_fused<1, 32>(a, s, name) : launch_fused<2, 32>(a, s, name);
+        if (a.dk == 64) return one ? launch_fused<1, 64>(a, s, name) : launch_fused<2, 64>(a, s, name);
+        return one ? launch_fused<1, 128>(a, s, name) : launch_fused<2, 128>(a, s, name);
     }
-    switch (a.dk) {
-    case 32: KNX_FUSED_NS(32)
-    case 64: KNX_FUSED_NS(64)
-    case 128:
-        switch (ns) {
-        case 1: return launch_fused<1, 128>(a, s, name);
-        case 2: return launch_fused<2, 128>(a, s, name);
-        default: return launch_fused<4, 128>(a, s, name);
-        }
-    default: return 1;
-    }
-#undef KNX_FUSED_NS
+    if (a.dk != a.dv || (!flash && !no_scratch(a) && !tiled_faster(a))) return 1;
+    const knx_flash_args f{a.Q, a.ldq, a.K, a.ldk, a.V, a.ldv, a.ctx, a.B, a.H, a.Rq, a.S, a.dk, a.scale, a.causal, 1.0f};
+    return knx_flash(f, s, name);
 }
 
 }  // namespace
@@ -305,6 +315,7 @@ extern "C" int knx_hip_attention_core_ex(const float* Q, int ldq, const float* K
     KNX_REQUIRE((long long)B * H * Rq * S <= (1LL << 40) && (long long)B * S * H * dv <= 0x7fffffffLL, name);
     hipStream_t s = knx::as_stream(stream);
     const AttnArgs a{Q, ldq, K, ldk, V, ldv, ctx, B, H, Rq, S, dk, dv, scale, causal};
+    KNX_REQUIRE(scores != nullptr || no_scratch(a), name);
     int rc = try_fused(a, s, name);
     if (rc != 1) return rc;
     KNX_REQUIRE(scores != nullptr, name);

@@ -14,42 +14,9 @@
 #include "knx_xgemm.hpp"
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte global access at any float address
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 namespace {
 
-// two fp32 values → two bf16 (round to nearest even) in one register
-__device__ __forceinline__ unsigned pk(float a, float b)
-{
-    const v2f v = {a, b};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, v2bf));
-}
-// what is left of a and b after their bf16 parts h (exact)
-__device__ __forceinline__ void rest(float& a, float& b, unsigned h)
-{
-    a = a - __builtin_bit_cast(float, h << 16);
-    b = b - __builtin_bit_cast(float, h & 0xffff0000u);
-}
-// four values into their three bf16 parts
-__device__ __forceinline__ void split4(float4 v, uint2& h, uint2& m, uint2& l)
-{
-    h = make_uint2(pk(v.x, v.y), pk(v.z, v.w));
-    rest(v.x, v.y, h.x);
-    rest(v.z, v.w, h.y);
-    m = make_uint2(pk(v.x, v.y), pk(v.z, v.w));
-    rest(v.x, v.y, m.x);
-    rest(v.z, v.w, m.y);
-    l = make_uint2(pk(v.x, v.y), pk(v.z, v.w));
-}
-
-__device__ __forceinline__ float4 load4(const float* p)
-{
-    const v4fu v = *reinterpret_cast<const v4fu*>(p);
-    return make_float4(v.x, v.y, v.z, v.w);
-}
 // up to four values at p, `left` of them inside the row
 __device__ __forceinline__ float4 load4_tail(const float* p, int left)
 {
@@ -61,16 +28,6 @@ __device__ __forceinline__ float4 load4_tail(const float* p, int left)
     return v;
 }
 
-// C = act(alpha·A·Bᵀ + bias) (+ R): BM×BN outputs per workgroup of WM×WN waves, K streamed 16 values at a time.  Rows of A
-// and B (any K, any float alignment) are loaded four values per lane, two k-tiles ahead, split into their bf16 parts by
-// the thread that loaded them (5.5 instructions per value, shared by every wave that multiplies it) and written to LDS
-// as MFMA fragments: 32 rows × 16 k of one part are 1 KB in lane order (lane = row + 32·(k / 8), 16 bytes each, the
-// upper half's rows exchanged by 8 so that the writes of four lanes per row spread over the banks).  Two LDS stages and
-// one barrier per k-tile: while the matrix cores work on one, the next is split and written.
-// What bounds it: at 4096³ and above the chip's power (1.9 GHz; 237 TFLOP/s of fp32 product are 1420 TFLOP/s of bf16,
-// where a plain bf16 GEMM of torch's reaches 1150 on the same card; fp32 instructions: 147 TFLOP/s); the smaller tiles
-// the split's instructions and the LDS, which overlap the multiplies only in part (128×128: 54% of the matrix cores'
-// cycles).  K-tiles of 32 or 64 values per barrier, four k-tiles of loads in flight and four waves of 64×64 were slower.
 // Where a row of A comes from: PLAIN a row of a matrix; CONV4, CONV1 an output pixel of a convolution (implicit GEMM: k
 // runs over (ky, kx, channel), the im2col row is gathered and never stored), four adjacent values of k being four
 // channels of one tap (CONV4, channels per group a multiple of 4) or anything (CONV1).
@@ -108,6 +65,16 @@ __device__ __forceinline__ const float* tap_at(const window& w, int2 e)
     return reinterpret_cast<const float*>((w.inside >> e.y) & 1 ? a : (unsigned long long)(uintptr_t)x_zeros);
 }
 
+// C = act(alpha·A·Bᵀ + bias) (+ R): BM×BN outputs per workgroup of WM×WN waves, K streamed 16 values at a time.  Rows of A
+// and B (any K, any float alignment) are loaded four values per lane, two k-tiles ahead, split into their bf16 parts by
+// the thread that loaded them (5.5 instructions per value, shared by every wave that multiplies it) and written to LDS
+// as MFMA fragments: 32 rows × 16 k of one part are 1 KB in lane order (lane = row + 32·(k / 8), 16 bytes each, the
+// upper half's rows at row ^ 12 so that the writes of four lanes per row spread over the banks).  Two LDS stages and
+// one barrier per k-tile: while the matrix cores work on one, the next is split and written.
+// What bounds it: at 4096³ and above the chip's power (1.9 GHz; 237 TFLOP/s of fp32 product are 1420 TFLOP/s of bf16,
+// where a plain bf16 GEMM of torch's reaches 1150 on the same card; fp32 instructions: 147 TFLOP/s); the smaller tiles
+// the split's instructions and the LDS, which overlap the multiplies only in part (128×128: 54% of the matrix cores'
+// cycles).  K-tiles of 32 or 64 values per barrier, four k-tiles of loads in flight and four waves of 64×64 were slower.
 template <int BM, int BN, int WM, int WN, int OCC, bool PIPE, int MODE>
 __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
 {
@@ -178,12 +145,12 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     // k-tile 0 is the odd one of K % KT values if there is one, the rest follow in order (tiles past the last repeat it:
     // loaded and written, never multiplied)
     auto gather4 = [&](const window& w, int k) __attribute__((always_inline)) {
-        if (MODE == CONV4) return load4(tap_at(w, taps[k >> 2]));
+        if (MODE == CONV4) return knx_load4(tap_at(w, taps[k >> 2]));
         return make_float4(*tap_at(w, taps[k]), *tap_at(w, taps[k + 1]), *tap_at(w, taps[k + 2]), *tap_at(w, taps[k + 3]));
     };
     auto gather4_tail = [&](const window& w, int k, int left) __attribute__((always_inline)) {
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (MODE == CONV4) return left > 0 ? load4(tap_at(w, taps[k >> 2])) : v;
+        if (MODE == CONV4) return left > 0 ? knx_load4(tap_at(w, taps[k >> 2])) : v;
         if (left > 0) v.x = *tap_at(w, taps[k]);
         if (left > 1) v.y = *tap_at(w, taps[k + 1]);
         if (left > 2) v.z = *tap_at(w, taps[k + 2]);
@@ -196,7 +163,7 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
 #pragma unroll
         for (int i = 0; i < P; ++i) {
             if (MODE != PLAIN && i < PA) v[i] = gather4(win[i], k + 4 * q);
-            else v[i] = load4((i < PA ? ta : tb) + k + off[i]);
+            else v[i] = knx_load4((i < PA ? ta : tb) + k + off[i]);
             __builtin_amdgcn_sched_barrier(0x3ff & ~0x30);  // loads stay in order
         }
     };
@@ -210,7 +177,7 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     };
     auto put = [&](int8_t* st, const float4& v, int i) __attribute__((always_inline)) {
         uint2 h, m, l;
-        split4(v, h, m, l);
+        knx_split4(v, h, m, l);
         *reinterpret_cast<uint2*>(st + woff[i]) = h;
         *reinterpret_cast<uint2*>(st + woff[i] + 1024) = m;
         *reinterpret_cast<uint2*>(st + woff[i] + 2048) = l;
@@ -233,18 +200,18 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
                 for (int e = 0; e < 16; ++e) accs[c][fi][fj][e] = 0.0f;
 
     constexpr int SA[6] = {2, 0, 1, 1, 0, 0}, SB[6] = {0, 2, 1, 0, 1, 0};  // the parts of A and of B, smallest product first
-    struct frags { v8bf a[FM][3], b[FN][3]; };
+    struct frags { knx_v8bf a[FM][3], b[FN][3]; };
     const int fa = wm * FM * 3072 + roff, fb = (BM / 32 + wn * FN) * 3072 + roff;
     auto fetch = [&](const int8_t* cur, frags& f) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
 #pragma unroll
-            for (int fi = 0; fi < FM; ++fi) f.a[fi][s] = *reinterpret_cast<const v8bf*>(cur + fa + fi * 3072 + s * 1024);
+            for (int fi = 0; fi < FM; ++fi) f.a[fi][s] = *reinterpret_cast<const knx_v8bf*>(cur + fa + fi * 3072 + s * 1024);
 #pragma unroll
-            for (int fj = 0; fj < FN; ++fj) f.b[fj][s] = *reinterpret_cast<const v8bf*>(cur + fb + fj * 3072 + s * 1024);
+            for (int fj = 0; fj < FN; ++fj) f.b[fj][s] = *reinterpret_cast<const knx_v8bf*>(cur + fb + fj * 3072 + s * 1024);
         }
     };
-    auto mfma = [&](const v8bf (&a)[3], const v8bf (&b)[3], int s, int fi, int fj) __attribute__((always_inline)) {
+    auto mfma = [&](const knx_v8bf (&a)[3], const knx_v8bf (&b)[3], int s, int fi, int fj) __attribute__((always_inline)) {
         accs[s % NA][fi][fj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[SA[s]], b[SB[s]], accs[s % NA][fi][fj], 0, 0, 0);
     };
     // PIPE: multiply the fragments f, read from LDS a k-tile ahead; meanwhile split and write the pieces in v to `nxt`
@@ -268,16 +235,16 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     };
     // otherwise (no registers for a second set of fragments): multiply the k-tile in `cur` a column of blocks at a time
     auto ktile = [&](const int8_t* cur, int8_t* nxt, const float4 (&v)[P]) __attribute__((always_inline)) {
-        v8bf a[FM][3];
+        knx_v8bf a[FM][3];
 #pragma unroll
         for (int fi = 0; fi < FM; ++fi)
 #pragma unroll
-            for (int s = 0; s < 3; ++s) a[fi][s] = *reinterpret_cast<const v8bf*>(cur + fa + fi * 3072 + s * 1024);
+            for (int s = 0; s < 3; ++s) a[fi][s] = *reinterpret_cast<const knx_v8bf*>(cur + fa + fi * 3072 + s * 1024);
 #pragma unroll
         for (int fj = 0; fj < FN; ++fj) {
-            v8bf b[3];
+            knx_v8bf b[3];
 #pragma unroll
-            for (int s = 0; s < 3; ++s) b[s] = *reinterpret_cast<const v8bf*>(cur + fb + fj * 3072 + s * 1024);
+            for (int s = 0; s < 3; ++s) b[s] = *reinterpret_cast<const knx_v8bf*>(cur + fb + fj * 3072 + s * 1024);
 #pragma unroll
             for (int s = 0; s < 6; ++s)
 #pragma unroll
