@@ -291,6 +291,14 @@ KNX_API int knx_hip_rnn_recurrence(int kind, int act, float alpha, int B, int T,
                                    const float* U, int u_nt, const int8_t* q, int kp, const float* qscale,
                                    const float* brec, float* h0, float* h1, float* dst, int stride, int ret_seq,
                                    void* scratch, size_t scratch_bytes, int* status, void* stream);
+/* The grid form for 65 to 256 rows: groups of at most 64 rows, each with workgroups and a barrier word of its own (rows of a
+ * recurrence never meet), at most 64 workgroups together in one launch.  Arguments and results as
+ * knx_hip_rnn_recurrence; scratch: 8 bytes per group of 64 rows.  Shapes _fits rejects are KNX_EINVAL. */
+KNX_API int knx_hip_rnn_recurrence_groups_fits(int kind, int B, int u, int i8);
+KNX_API int knx_hip_rnn_recurrence_groups(int kind, int act, float alpha, int B, int T, int u, int dir, const float* zx,
+                                          const float* U, int u_nt, const int8_t* q, int kp, const float* qscale,
+                                          const float* brec, float* h0, float* h1, float* dst, int stride, int ret_seq,
+                                          void* scratch, size_t scratch_bytes, int* status, void* stream);
 
 #ifdef __cplusplus
 }

@@ -9,7 +9,7 @@
 // against 5.7 and 17 µs with device-scope fences in every thread.
 //
 // Counting: one 64-bit word per barrier, zero (or a multiple of 256) before the first launch.  Every launch adds
-// exactly 256 to each word: every workgroup 1, workgroup 0 also the 256 − G that the grid lacks.  A workgroup's
+// exactly 256 to each word it uses: every workgroup 1, workgroup 0 also the 256 − G that the G of them lack.  A workgroup's
 // own atomic add returns the word before it, so the word's value at the end of this barrier is the next multiple
 // of 256, and the workgroup waits (polling) until the word reaches it.  Words are never reset and never need to be:
 // launches on one scratch are ordered by their stream, and 2^64 / 256 launches do not wrap.  The wait is bounded:
@@ -34,13 +34,14 @@ struct GridSync {
     unsigned spin;              // polls before a workgroup stops waiting
 };
 
-__device__ __forceinline__ void grid_barrier(const GridSync& gs, unsigned b)
+// Barrier word b, of `count` workgroups of the launch of which this one is number `index` (all of them by default).
+__device__ __forceinline__ void grid_barrier(const GridSync& gs, unsigned b, unsigned index, unsigned count)
 {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's device-scope stores are complete
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long* w = gs.words + b;
-        const unsigned long long add = blockIdx.x == 0 ? KNX_GRID_QUANTUM - gridDim.x + 1 : 1;
+        const unsigned long long add = index == 0 ? KNX_GRID_QUANTUM - count + 1 : 1;
         const unsigned long long old = __hip_atomic_fetch_add(w, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned long long target = (old / KNX_GRID_QUANTUM + 1) * KNX_GRID_QUANTUM;
         if (old + add < target) {
@@ -58,6 +59,11 @@ __device__ __forceinline__ void grid_barrier(const GridSync& gs, unsigned b)
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
+}
+
+__device__ __forceinline__ void grid_barrier(const GridSync& gs, unsigned b)
+{
+    grid_barrier(gs, b, blockIdx.x, gridDim.x);
 }
 
 }  // namespace knx

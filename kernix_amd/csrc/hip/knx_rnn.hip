@@ -33,11 +33,12 @@
 namespace {
 
 constexpr int kThreads = 256, kWaves = 4;
-constexpr int kMaxPairs = 2;             // (row, unit) pairs per thread in the cell phase: B·uw ≤ 512
+constexpr int kGroupRows = 64;           // rows of a group of workgroups
+constexpr int kMaxGroups = 4;
 constexpr int kMaxGrid = 64;
 constexpr int kLoads = 8;                // float4 loads of h in flight per thread
 constexpr int kMaxUnits = 2048;          // the multi-workgroup kernel: a row of h is at most kLoads float4s per lane
-constexpr size_t kMaxLds = 120 * 1024;
+constexpr size_t kMaxLds = 120 * 1024, kMaxLdsGroups = 156 * 1024;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -57,6 +58,7 @@ struct RnnArgs {
     float* h1;
     float* dst;
     knx::GridSync gs;
+    int rg, gw;           // rows and workgroups of a group (rnn_recurrence)
     // the row-split kernel only: the LINEAR step that reads only the last state, at the end of the same launch
     // (dn > 0): y = act(h_T·Wᵀ + b) over dn outputs, int8 (dq: dn rows of dkp bytes, dqs their scales) or fp32 (dw:
     // dn rows of u floats); dy: B rows of dn
@@ -112,7 +114,10 @@ __host__ __device__ inline Lds lds_layout(int B, int gates, int uw, int up, bool
 // and the activation's switch resolved at compile time a timestep's cells took 0.46 against 0.70 µs.
 constexpr int kActAny = -100;
 
-template <bool I8, int KIND, int ACT>
+// MP: (row, unit) pairs per thread in the cell phase, rows of a group · uw ≤ MP · kThreads.
+// More than 64 rows: groups of at most 64, each with workgroups and a barrier word of its own (the rows of a recurrence
+// never meet), all in the one launch.  LSTM, 100 rows, u = 200, 32 timesteps: see knx_hip_rnn_recurrence_fits.
+template <bool I8, int KIND, int ACT, int MP>
 __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -121,11 +126,16 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
     const int act = ACT == kActAny ? a.act : ACT;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // the same value, known to the compiler as uniform
-    const int B = a.B, T = a.T, u = a.u, up = a.up, gu = a.gu, G = a.gates, ldh = a.ldh;
-    const int j0 = blockIdx.x * a.uw;
-    const int nwu = min(a.uw, u - j0);  // ≥ 1: the grid has ⌈u / uw⌉ workgroups
+    const int group = (int)blockIdx.x / a.gw, member = (int)blockIdx.x % a.gw, row0 = group * a.rg;
+    const int B = min(a.rg, a.B - row0), T = a.T, u = a.u, up = a.up, gu = a.gu, G = a.gates, ldh = a.ldh;
+    a.zx += (size_t)row0 * T * gu;
+    a.h0 += (size_t)row0 * ldh;
+    a.h1 += (size_t)row0 * ldh;
+    a.dst += (size_t)row0 * (a.ret_seq ? T : 1) * a.stride;
+    const int j0 = member * a.uw;
+    const int nwu = min(a.uw, u - j0);  // ≥ 1: a group has ⌈u / uw⌉ workgroups
     const int NC = G * nwu, NCM = G * a.uw;
-    const Lds L = lds_layout(B, G, a.uw, up, i8, h32);
+    const Lds L = lds_layout(a.rg, G, a.uw, up, i8, h32);
     const int upp = L.upp, hp = L.hp, hwp = L.hwp, ncp = L.ncp;
     float* usf = reinterpret_cast<float*>(smem + L.us);
     int* usw = reinterpret_cast<int*>(smem + L.us);
@@ -170,8 +180,8 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
     }
     // this thread's (row, unit) pairs of the cell phase and their per-column constants
     const int npairs = B * nwu;
-    float cst[kMaxPairs];
-    for (int i = 0; i < kMaxPairs; ++i) cst[i] = 0.0f;
+    float cst[MP];
+    for (int i = 0; i < MP; ++i) cst[i] = 0.0f;
 
     // loading h_{t−1}: a row is W4 float4s over LR lanes (a power of two: as many as keep every row within one pass
     // of the four waves, at least enough for kLoads float4s per lane to cover the row, at most one per float4), RPW
@@ -190,10 +200,10 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
     const int nkc = i8 ? up / 64 : up / 16;
 
     // the input-side gate values of this thread's pairs, one timestep ahead (they do not depend on h)
-    auto load_z = [&](int st, float (&z)[kMaxPairs][4]) {
+    auto load_z = [&](int st, float (&z)[MP][4]) {
         const int tt = a.dir ? T - 1 - st : st;
 #pragma unroll
-        for (int i = 0; i < kMaxPairs; ++i) {
+        for (int i = 0; i < MP; ++i) {
             const int pr = tid + kThreads * i;
             const int b = pr / nwu, jj = pr % nwu;
 #pragma unroll
@@ -209,15 +219,15 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
         r[b * NCM + cc] = x;
     };
     __syncthreads();
-    float zn[kMaxPairs][4];
+    float zn[MP][4];
     load_z(0, zn);
     for (int step = 0; step < T; ++step) {
         const int t = a.dir ? T - 1 - step : step;
         const float* hin = (step & 1) ? a.h0 : a.h1;  // h_{t−1}: written at the previous step
         float* hout = (step & 1) ? a.h1 : a.h0;
-        float zv[kMaxPairs][4];
+        float zv[MP][4];
 #pragma unroll
-        for (int i = 0; i < kMaxPairs; ++i)
+        for (int i = 0; i < MP; ++i)
 #pragma unroll
             for (int g = 0; g < 4; ++g) zv[i][g] = zn[i][g];
         if (step + 1 < T) load_z(step + 1, zn);
@@ -358,7 +368,7 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
         }
         // the cells
 #pragma unroll
-        for (int i = 0; i < kMaxPairs; ++i) {
+        for (int i = 0; i < MP; ++i) {
             const int pr = tid + kThreads * i;
             if (pr >= npairs) continue;
             const int b = pr / nwu, jj = pr % nwu, j = j0 + jj;
@@ -384,7 +394,7 @@ __global__ void __launch_bounds__(kThreads) rnn_recurrence(RnnArgs a)
             if (a.ret_seq) a.dst[((size_t)b * T + t) * a.stride + j] = hv;
             else if (step + 1 == T) a.dst[(size_t)b * a.stride + j] = hv;
         }
-        if (step + 1 < T) knx::grid_barrier(a.gs, 0);  // also: every thread is done with hs and r of this step
+        if (step + 1 < T) knx::grid_barrier(a.gs, group, member, a.gw);  // also: every thread is done with hs and r of this step
     }
 }
 
@@ -701,16 +711,33 @@ int solo_lanes(int B, int gu, int u, bool i8)
 // units per workgroup: enough that the workgroup's gate columns fill a 16-wide tile of the products (LSTM 4, GRU 5,
 // simple RNN 16 units), more where u needs it to stay within kMaxGrid workgroups, fewer where the (row, unit) pairs
 // would not fit the threads
-int units_per_wg(int B, int u, int gates)
+struct GridSplit {
+    int groups, rg, gw, uw;  // groups of rg rows, each gw workgroups of uw units
+};
+GridSplit grid_split(int B, int u, int gates)
 {
-    const int least = (u + kMaxGrid - 1) / kMaxGrid;
-    int uw = std::max(least, 16 / gates);
+    GridSplit p;
+    p.groups = (B + kGroupRows - 1) / kGroupRows;
+    p.rg = (B + p.groups - 1) / p.groups;
+    const int most = std::max(1, kMaxGrid / p.groups), least = (u + most - 1) / most;
+    p.uw = std::max(least, 16 / gates);
     if (const char* e = getenv("KNX_RNN_UNITS")) {  // tuning: units per workgroup
         const int v = atoi(e);
-        if (v >= 1) uw = std::max(least, v);
+        if (v >= 1) p.uw = std::max(least, v);
     }
-    while (B * uw > kThreads * kMaxPairs && uw > least) --uw;
-    return uw;
+    while (p.rg * p.uw > kThreads * 2 && p.uw > least) --p.uw;
+    p.gw = (u + p.uw - 1) / p.uw;
+    return p;
+}
+
+template <bool I8, int KIND, int ACT, int MP>
+int launch_grid(const RnnArgs& a, int G, size_t lds, hipStream_t s, const char* name)
+{
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&rnn_recurrence<I8, KIND, ACT, MP>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLdsGroups);
+    if (attr != hipSuccess) return knx::fail(KNX_EHIP, "%s: %s", name, hipGetErrorString(attr));
+    hipLaunchKernelGGL((rnn_recurrence<I8, KIND, ACT, MP>), dim3((unsigned)G), dim3(kThreads), lds, s, a);
+    return knx::check_launch(name);
 }
 
 // one launch of the instantiation for (I8, KIND, ACT): the row-split kernel when ks > 0, else the grid of G
@@ -724,11 +751,7 @@ int launch_rnn(const RnnArgs& a, int ks, int G, size_t lds, hipStream_t s, const
                            ks, R);
         return knx::check_launch(name);
     }
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&rnn_recurrence<I8, KIND, ACT>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
-    if (attr != hipSuccess) return knx::fail(KNX_EHIP, "%s: %s", name, hipGetErrorString(attr));
-    hipLaunchKernelGGL((rnn_recurrence<I8, KIND, ACT>), dim3((unsigned)G), dim3(kThreads), lds, s, a);
-    return knx::check_launch(name);
+    return a.rg * a.uw <= 2 * kThreads ? launch_grid<I8, KIND, ACT, 2>(a, G, lds, s, name) : launch_grid<I8, KIND, ACT, 4>(a, G, lds, s, name);
 }
 
 template <bool I8, int KIND>
@@ -752,10 +775,19 @@ extern "C" int knx_hip_rnn_recurrence_fits(int kind, int B, int u, int i8)
     if ((kind != 4 && kind != 5 && kind != 6) || B < 1 || u < 1 || u > 65536) return 0;
     const int gates = kind == 4 ? 4 : kind == 5 ? 3 : 1;
     if (solo_lanes(B, gates * u, u, i8 != 0) > 0) return 1;
-    if (B > 64 || u > kMaxUnits) return 0;
-    const int uw = units_per_wg(B, u, gates);
-    if ((u + uw - 1) / uw > kMaxGrid || B * uw > kThreads * kMaxPairs) return 0;
-    return lds_layout(B, gates, uw, k_extent(u, i8 != 0), i8 != 0, !i8 || kind == 5).total <= kMaxLds ? 1 : 0;
+    if (B > kGroupRows || u > kMaxUnits) return 0;
+    const GridSplit p = grid_split(B, u, gates);
+    if (p.gw > kMaxGrid || B * p.uw > kThreads * 2) return 0;
+    return lds_layout(B, gates, p.uw, k_extent(u, i8 != 0), i8 != 0, !i8 || kind == 5).total <= kMaxLds ? 1 : 0;
+}
+
+extern "C" int knx_hip_rnn_recurrence_groups_fits(int kind, int B, int u, int i8)
+{
+    if ((kind != 4 && kind != 5 && kind != 6) || B <= kGroupRows || B > kGroupRows * kMaxGroups || u < 1 || u > kMaxUnits) return 0;
+    const int gates = kind == 4 ? 4 : kind == 5 ? 3 : 1;
+    const GridSplit p = grid_split(B, u, gates);
+    if (p.groups * p.gw > kMaxGrid || p.rg * p.uw > kThreads * 4) return 0;
+    return lds_layout(p.rg, gates, p.uw, k_extent(u, i8 != 0), i8 != 0, !i8 || kind == 5).total <= kMaxLdsGroups ? 1 : 0;
 }
 
 extern "C" int knx_hip_rnn_recurrence_dense_fits(int kind, int B, int u, int i8, int n)
@@ -785,7 +817,7 @@ extern "C" int knx_hip_rnn_recurrence_dense(int kind, int act, float alpha, int 
     RnnArgs a{};
     a.kind = kind; a.act = act; a.alpha = alpha;
     a.B = B; a.T = T; a.u = u; a.gu = gates * u; a.gates = gates; a.dir = dir; a.ret_seq = 0;
-    a.stride = stride; a.uw = units_per_wg(B, u, gates);
+    a.stride = stride;
     a.up = k_extent(u, q != nullptr); a.ldh = (u + 3) / 4 * 4;
     a.zx = zx; a.U = U; a.u_nt = u_nt != 0; a.q = q; a.kp = kp; a.qs = qscale; a.brec = brec;
     a.dst = dst;
@@ -797,6 +829,37 @@ extern "C" int knx_hip_rnn_recurrence_dense(int kind, int act, float alpha, int 
     return launch_kind<false>(a, ks, 0, 0, s, name);
 }
 
+// both recurrences over the sequence: ks > 0 the rows split over workgroups that hold all of U, else the grid
+static int recurrence(int kind, int act, float alpha, int B, int T, int u, int dir, const float* zx, const float* U,
+                      int u_nt, const int8_t* q, int kp, const float* qscale, const float* brec, float* h0, float* h1,
+                      float* dst, int stride, int ret_seq, void* scratch, size_t scratch_bytes, int* status, int ks,
+                      void* stream, const char* name)
+{
+    const int gates = kind == 4 ? 4 : kind == 5 ? 3 : 1;
+    KNX_REQUIRE(zx != nullptr && h0 != nullptr && h1 != nullptr && dst != nullptr && stride >= u, name);
+    KNX_REQUIRE((((uintptr_t)h0 | (uintptr_t)h1) & 15) == 0, name);
+    KNX_REQUIRE(kind != 5 || brec != nullptr, name);
+    KNX_REQUIRE(q != nullptr ? (qscale != nullptr && kp >= (u + 3) / 4 * 4 && ((uintptr_t)q & 3) == 0 && kp % 4 == 0)
+                             : U != nullptr, name);
+    KNX_REQUIRE(scratch != nullptr && ((uintptr_t)scratch & 255) == 0 && scratch_bytes >= 8 * (size_t)((B + kGroupRows - 1) / kGroupRows), name);
+    KNX_REQUIRE(status != nullptr && ((uintptr_t)status & 3) == 0, name);
+    RnnArgs a{};
+    a.kind = kind; a.act = act; a.alpha = alpha;
+    a.B = B; a.T = T; a.u = u; a.gu = gates * u; a.gates = gates; a.dir = dir; a.ret_seq = ret_seq != 0;
+    a.stride = stride;
+    const GridSplit p = grid_split(B, u, gates);
+    a.uw = p.uw; a.rg = p.rg; a.gw = p.gw;
+    a.up = k_extent(u, q != nullptr); a.ldh = (u + 3) / 4 * 4;
+    a.zx = zx; a.U = U; a.u_nt = u_nt != 0; a.q = q; a.kp = kp; a.qs = qscale; a.brec = brec;
+    a.h0 = h0; a.h1 = h1; a.dst = dst;
+    a.gs = knx::GridSync{static_cast<unsigned long long*>(scratch), status, knx::grid_spin_limit()};
+    const int G = p.groups * p.gw;
+    const size_t lds = ks > 0 ? 0 : lds_layout(p.rg, gates, a.uw, a.up, q != nullptr, q == nullptr || kind == 5).total;
+    const hipStream_t s = knx::as_stream(stream);
+    if (q != nullptr) return launch_kind<true>(a, ks, G, lds, s, name);
+    return launch_kind<false>(a, ks, G, lds, s, name);
+}
+
 extern "C" int knx_hip_rnn_recurrence(int kind, int act, float alpha, int B, int T, int u, int dir, const float* zx,
                                       const float* U, int u_nt, const int8_t* q, int kp, const float* qscale,
                                       const float* brec, float* h0, float* h1, float* dst, int stride, int ret_seq,
@@ -806,26 +869,20 @@ extern "C" int knx_hip_rnn_recurrence(int kind, int act, float alpha, int B, int
     KNX_ENTRY(name);
     KNX_REQUIRE(T >= 1 && act >= -1 && act <= 15 && (dir == 0 || dir == 1), name);
     KNX_REQUIRE(knx_hip_rnn_recurrence_fits(kind, B, u, q != nullptr), name);
-    const int gates = kind == 4 ? 4 : kind == 5 ? 3 : 1;
-    KNX_REQUIRE(zx != nullptr && h0 != nullptr && h1 != nullptr && dst != nullptr && stride >= u, name);
-    KNX_REQUIRE((((uintptr_t)h0 | (uintptr_t)h1) & 15) == 0, name);
-    KNX_REQUIRE(kind != 5 || brec != nullptr, name);
-    KNX_REQUIRE(q != nullptr ? (qscale != nullptr && kp >= (u + 3) / 4 * 4 && ((uintptr_t)q & 3) == 0 && kp % 4 == 0)
-                             : U != nullptr, name);
-    KNX_REQUIRE(scratch != nullptr && ((uintptr_t)scratch & 255) == 0 && scratch_bytes >= 8, name);
-    KNX_REQUIRE(status != nullptr && ((uintptr_t)status & 3) == 0, name);
-    RnnArgs a{};
-    a.kind = kind; a.act = act; a.alpha = alpha;
-    a.B = B; a.T = T; a.u = u; a.gu = gates * u; a.gates = gates; a.dir = dir; a.ret_seq = ret_seq != 0;
-    a.stride = stride; a.uw = units_per_wg(B, u, gates);
-    a.up = k_extent(u, q != nullptr); a.ldh = (u + 3) / 4 * 4;
-    a.zx = zx; a.U = U; a.u_nt = u_nt != 0; a.q = q; a.kp = kp; a.qs = qscale; a.brec = brec;
-    a.h0 = h0; a.h1 = h1; a.dst = dst;
-    a.gs = knx::GridSync{static_cast<unsigned long long*>(scratch), status, knx::grid_spin_limit()};
-    const int ks = solo_lanes(B, a.gu, u, q != nullptr);
-    const int G = (u + a.uw - 1) / a.uw;
-    const size_t lds = ks > 0 ? 0 : lds_layout(B, gates, a.uw, a.up, q != nullptr, q == nullptr || kind == 5).total;
-    const hipStream_t s = knx::as_stream(stream);
-    if (q != nullptr) return launch_kind<true>(a, ks, G, lds, s, name);
-    return launch_kind<false>(a, ks, G, lds, s, name);
+    const int ks = solo_lanes(B, (kind == 4 ? 4 : kind == 5 ? 3 : 1) * u, u, q != nullptr);
+    return recurrence(kind, act, alpha, B, T, u, dir, zx, U, u_nt, q, kp, qscale, brec, h0, h1, dst, stride, ret_seq,
+                      scratch, scratch_bytes, status, ks, stream, name);
+}
+
+extern "C" int knx_hip_rnn_recurrence_groups(int kind, int act, float alpha, int B, int T, int u, int dir, const float* zx,
+                                             const float* U, int u_nt, const int8_t* q, int kp, const float* qscale,
+                                             const float* brec, float* h0, float* h1, float* dst, int stride, int ret_seq,
+                                             void* scratch, size_t scratch_bytes, int* status, void* stream)
+{
+    const char* name = "knx_hip_rnn_recurrence_groups";
+    KNX_ENTRY(name);
+    KNX_REQUIRE(T >= 1 && act >= -1 && act <= 15 && (dir == 0 || dir == 1), name);
+    KNX_REQUIRE(knx_hip_rnn_recurrence_groups_fits(kind, B, u, q != nullptr), name);
+    return recurrence(kind, act, alpha, B, T, u, dir, zx, U, u_nt, q, kp, qscale, brec, h0, h1, dst, stride, ret_seq,
+                      scratch, scratch_bytes, status, 0, stream, name);
 }

@@ -605,12 +605,14 @@ static int run_rnn_dir(const kernix_model* m, kernix_step* s, int dir, const flo
                                                    dense->alpha, dense->y, st),
                       "RNN recurrence + Linear");
     }
-    if (rnn_persistent(m) && knx_hip_rnn_recurrence_fits(kind, B, u, i8)) {
+    const int one = rnn_persistent(m) && knx_hip_rnn_recurrence_fits(kind, B, u, i8);
+    if (one || (rnn_persistent(m) && knx_hip_rnn_recurrence_groups_fits(kind, B, u, i8))) {
         /* every timestep in one launch; h alternates between h and the recurrent-term buffer (B rows of u4 each) */
         if (!i8 && U == NULL) return -1;
-        return hip_ok(knx_hip_rnn_recurrence(kind, s->act, s->alpha, B, T, u, dir, zx, i8 ? NULL : U, q != NULL,
-                                             i8 ? dq : NULL, q != NULL ? q->kp : 0, dsc, brec, h, hu, dst, stride,
-                                             s->ret_seq, m->dev->chain, m->dev->chain_bytes, m->dev->chain_status, st),
+        return hip_ok((one ? knx_hip_rnn_recurrence : knx_hip_rnn_recurrence_groups)(
+                          kind, s->act, s->alpha, B, T, u, dir, zx, i8 ? NULL : U, q != NULL, i8 ? dq : NULL,
+                          q != NULL ? q->kp : 0, dsc, brec, h, hu, dst, stride, s->ret_seq, m->dev->chain,
+                          m->dev->chain_bytes, m->dev->chain_status, st),
                       "RNN recurrence");
     }
     for (int step = 0; step < T; step++) {

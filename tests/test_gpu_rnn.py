@@ -269,3 +269,36 @@ def test_recurrence_that_stopped_waiting_is_recomputed(tmp_path, monkeypatch):
     monkeypatch.setenv("KNX_GRID_SPIN", "0")
     got = forward(p, x, "i8", monkeypatch, True, solo=False)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("cell,units,dirs", [("LSTM", 200, 1), ("LSTM", 256, 1), ("GRU", 161, 2), ("GRU", 256, 1), ("RNN", 300, 2)])
+@pytest.mark.parametrize("int8,mode", [(False, "ref"), (True, "ref"), (True, "i8")])
+@pytest.mark.parametrize("batch", [65, 100, 129, 193, 256])
+def test_groups_of_rows(tmp_path, monkeypatch, cell, units, dirs, int8, mode, batch):
+    """65 to 256 rows of more units than a workgroup holds: groups of up to 64 rows in one launch (uneven last groups, four
+    pairs of row and unit per thread), against one launch per timestep: the same bits for int8 recurrences"""
+    i8 = int8 and mode == "i8"
+    L = hipabi.lib()
+    kind = {"LSTM": 4, "GRU": 5, "RNN": 6}[cell]
+    if not i8 and cell != "RNN":
+        assert L.knx_hip_rnn_recurrence_fits(kind, batch, units, int(i8)) == 0
+    p = str(tmp_path / "r.knx")
+    x = configs.lstm(p, seed=batch, batch=batch, T=5, fin=24, units=units, int8=int8, cell=cell, directions=dirs)
+    got = forward(p, x, mode, monkeypatch, True)
+    per_step = forward(p, x, mode, monkeypatch, False)
+    if i8:
+        assert np.array_equal(got, per_step)
+    else:
+        assert rel_err(got, per_step) <= 1e-5
+
+
+def test_groups_of_rows_run_and_recover(tmp_path, monkeypatch):
+    """the forward takes the groups' entry point, and with a poll limit of 0 it is recomputed one launch per timestep"""
+    p = str(tmp_path / "g.knx")
+    x = configs.lstm(p, seed=4, batch=150, T=6, fin=16, units=200, int8=True)
+    want = forward(p, x, "i8", monkeypatch, False)
+    monkeypatch.setenv("KNX_GRID_SPIN", "0")
+    assert np.array_equal(forward(p, x, "i8", monkeypatch, True), want)
+    monkeypatch.setenv("KNX_HIP_FAIL", "knx_hip_rnn_recurrence_groups")
+    with pytest.raises(RuntimeError):
+        forward(p, x, "i8", monkeypatch, True)
