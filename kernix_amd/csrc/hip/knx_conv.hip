@@ -424,6 +424,112 @@ int conv_small_entry(const knx_conv_geom* g, const float* x, const float* w, boo
     return knx::check_launch(name);
 }
 
+// ---------------------------------------------------------------- depthwise convolution
+// One filter per channel (groups = C = Co) is no contraction: an output is kh·kw multiply-adds of its own channel, and as
+// one GEMM of a single column per group it ran 31 of 32 matrix lanes empty (217 images of 8×8×174: 296 µs for 19 MB).
+// Here a thread takes one output pixel of four channels (VEC: C a multiple of 4, 16-byte aligned) or of one, consecutive
+// threads consecutive channels; the weights are staged once per workgroup in LDS, tap-major.  Bounded by memory: the
+// taps a pixel shares with its neighbours come from the caches.
+struct DepthArgs {
+    knx_conv_geom g;
+    const float* x;
+    const float* w;
+    const float* bias;
+    const float* R;
+    float* y;
+    int act;
+    float alpha;
+    int wsc, wsk;  // weight (channel c, tap k) at w[c·wsc + k·wsk]
+    unsigned n;    // outputs, in units of four channels or one
+};
+
+template <bool VEC, int TAPS>  // TAPS: kh·kw if known (9), else 0
+__global__ void __launch_bounds__(256) conv_depthwise(DepthArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) float ws[];  // [tap][channel]
+    const knx_conv_geom& g = a.g;
+    const int C = g.C, taps = TAPS ? TAPS : g.kh * g.kw;
+    for (int i = threadIdx.x; i < taps * C; i += 256) {
+        const int c = a.wsk == 1 ? i / taps : i % C, k = a.wsk == 1 ? i % taps : i / C;  // i walks the weight in memory order
+        ws[k * C + c] = a.w[(size_t)c * a.wsc + (size_t)k * a.wsk];
+    }
+    __syncthreads();
+    constexpr int V = VEC ? 4 : 1;
+    const unsigned cv = (unsigned)C / V;
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256) {
+        const unsigned pix = i / cv, c = (i - pix * cv) * V;
+        const unsigned row = pix / g.Wo;
+        const int ox = (int)(pix - row * g.Wo), oy = (int)(row % g.Ho), b = (int)(row / g.Ho);
+        const int iy = oy * g.sh - g.pt, ix = ox * g.sw - g.pl;
+        const float* px = a.x + ((long long)b * g.H * g.W) * C + c;
+        float acc[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] = 0.0f;
+        auto tap = [&](int k, int ky, int kx) __attribute__((always_inline)) {
+            const int yy = iy + ky * g.dh, xx = ix + kx * g.dw;
+            const bool in = (unsigned)yy < (unsigned)g.H && (unsigned)xx < (unsigned)g.W;
+            if (!in) return;
+            const float* src = px + ((long long)yy * g.W + xx) * C;
+            float xv[V], wv[V];
+            if (VEC) {
+                *reinterpret_cast<float4*>(xv) = *reinterpret_cast<const float4*>(src);
+                *reinterpret_cast<float4*>(wv) = *reinterpret_cast<const float4*>(ws + k * C + c);
+            } else {
+                xv[0] = *src;
+                wv[0] = ws[k * C + c];
+            }
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[v] = __builtin_fmaf(xv[v], wv[v], acc[v]);
+        };
+        if (TAPS == 9) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k) tap(k, k / 3, k % 3);
+        } else {
+            for (int ky = 0, k = 0; ky < g.kh; ++ky)
+                for (int kx = 0; kx < g.kw; ++kx, ++k) tap(k, ky, kx);
+        }
+        const size_t o = (size_t)pix * C + c;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if (a.bias) acc[v] = acc[v] + a.bias[c + v];
+            acc[v] = a.act == -1 ? acc[v] : a.act == 0 ? (acc[v] >= 0.0f ? acc[v] : 0.0f) : knx_act(acc[v], a.act, a.alpha);
+        }
+        if (VEC) {
+            float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (a.R) r = *reinterpret_cast<const float4*>(a.R + o);
+            if (a.R)
+#pragma unroll
+                for (int v = 0; v < V; ++v) acc[v] = acc[v] + (&r.x)[v];
+            *reinterpret_cast<float4*>(a.y + o) = *reinterpret_cast<const float4*>(acc);
+        } else {
+            a.y[o] = a.R ? acc[0] + a.R[o] : acc[0];
+        }
+    }
+}
+
+// 1 without launching where the shape is another one (more filters per channel, weights past 64 KB of LDS, 2^31 outputs)
+int depthwise_entry(const knx_conv_geom* g, const float* x, const float* w, bool transposed, const float* bias, int act,
+                    float alpha, const float* R, float* y, hipStream_t s, const char* name)
+{
+    const long long taps = (long long)g->kh * g->kw, n = (long long)g->B * g->Ho * g->Wo * g->C;
+    if (g->groups != g->C || g->Co != g->C || g->C < 2 || taps * g->C * 4 > 65536 || n > 0x7fffffffLL) return 1;
+    DepthArgs a{};
+    a.g = *g; a.x = x; a.w = w; a.bias = bias; a.R = R; a.y = y; a.act = act; a.alpha = alpha;
+    a.wsc = transposed ? (int)taps : 1;
+    a.wsk = transposed ? 1 : g->Co;
+    const bool vec = g->C % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)R) & 15) == 0;
+    a.n = (unsigned)(vec ? n / 4 : n);
+    // a workgroup stages all weights: enough workgroups to fill the chip, several outputs per thread beyond
+    const unsigned blocks = (unsigned)std::min<long long>((a.n + 255) / 256, 8LL * knx::num_cus());
+    const unsigned lds = (unsigned)(taps * g->C * 4);
+    const bool nine = g->kh == 3 && g->kw == 3;
+    if (vec && nine) hipLaunchKernelGGL((conv_depthwise<true, 9>), dim3(blocks), dim3(256), lds, s, a);
+    else if (vec) hipLaunchKernelGGL((conv_depthwise<true, 0>), dim3(blocks), dim3(256), lds, s, a);
+    else if (nine) hipLaunchKernelGGL((conv_depthwise<false, 9>), dim3(blocks), dim3(256), lds, s, a);
+    else hipLaunchKernelGGL((conv_depthwise<false, 0>), dim3(blocks), dim3(256), lds, s, a);
+    return knx::check_launch(name);
+}
+
 template <int BM, int BN, int WM, int WN, bool TB>
 int launch(ConvArgs p, bool vec, hipStream_t s, const char* name)
 {
@@ -451,6 +557,10 @@ int conv_entry(const knx_conv_geom* g, const float* x, const float* w, const flo
     hipStream_t s = knx::as_stream(stream);
     {
         const int rc = conv_small_entry(g, x, w, TB, bias, act, R, y, s, name);
+        if (rc != 1) return rc;
+    }
+    {
+        const int rc = depthwise_entry(g, x, w, TB, bias, act, alpha, R, y, s, name);
         if (rc != 1) return rc;
     }
     if (TB) {

@@ -474,20 +474,20 @@ int pick_tile(const knx_xargs& p, int batch, bool conv, float* us)
 {
     static const struct {
         int tile, bm, bn;
-        float idle, busy, fixed;
-    } T[] = {{KNX_X256x256, 256, 256, 1.58f, 2.2f, 18.0f},
-             {KNX_X256x128, 256, 128, 0.78f, 1.15f, 10.0f},
-             {KNX_X256x64, 256, 64, 0.78f, 0.65f, 9.0f},
-             {KNX_X128x128, 128, 128, 0.41f, 0.63f, 8.0f},
-             {KNX_X128x64, 128, 64, 0.37f, 0.37f, 7.5f},
-             {KNX_X64x64, 64, 64, 0.26f, 0.21f, 7.0f}};
+        float idle, busy, fixed, windows;  // windows: µs for a convolution's tap windows and table before the first load
+    } T[] = {{KNX_X256x256, 256, 256, 1.58f, 2.2f, 18.0f, 0.0f},
+             {KNX_X256x128, 256, 128, 0.78f, 1.15f, 10.0f, 3.5f},
+             {KNX_X256x64, 256, 64, 0.78f, 0.65f, 9.0f, 4.0f},
+             {KNX_X128x128, 128, 128, 0.41f, 0.63f, 8.0f, 2.0f},
+             {KNX_X128x64, 128, 64, 0.37f, 0.37f, 7.5f, 5.0f},
+             {KNX_X64x64, 64, 64, 0.26f, 0.21f, 7.0f, 1.5f}};
     int best = KNX_X64x64;
     *us = 0.0f;
     for (const auto& t : T) {
         if (conv && t.tile == KNX_X256x256) continue;
         const long tiles = (long)((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * batch, cus = knx::num_cus();
         const long rounds = (tiles + cus - 1) / cus;
-        const float e = t.fixed + (float)p.K / 16.0f * (2 * tiles <= cus ? t.idle : t.busy * (float)rounds);
+        const float e = t.fixed + (conv ? t.windows : 0.0f) + (float)p.K / 16.0f * (2 * tiles <= cus ? t.idle : t.busy * (float)rounds);
         if (*us == 0.0f || e < *us) *us = e, best = t.tile;
     }
     return best;

@@ -129,3 +129,39 @@ def test_convolution(L, C, Co, k, stride, dil, groups, tile, monkeypatch):
         assert np.array_equal(part[inf], want[inf])
         lim = bound(torch.nan_to_num(A, posinf=0.0).numpy(), B.numpy(), 16 * K)
         assert np.all(np.abs(part[ok] - want[ok]) <= lim[ok])
+
+
+@pytest.mark.parametrize("B,H,W,C,k,stride,dil,pad", [(2, 9, 7, 4, 3, 1, 1, 1), (3, 14, 14, 174, 3, 2, 1, 1), (1, 5, 6, 3, 3, 1, 2, 2),
+                                                      (2, 12, 11, 64, 5, 1, 1, 2), (1, 8, 8, 6, 7, 2, 1, 3), (2, 3, 3, 2, 1, 1, 1, 0),
+                                                      (40, 33, 31, 132, 3, 1, 1, 1)])
+@pytest.mark.parametrize("transposed,act,res", [(True, 0, False), (True, -1, True), (False, 1, False)])
+def test_depthwise(L, B, H, W, C, k, stride, dil, pad, transposed, act, res):
+    """one filter per channel, four channels per thread or one, both weight layouts, the residual in place; a rounding per
+    multiply-add and a few for the epilogue (GELU: its polynomial's 1.5e-7 and the hardware exp2 and reciprocal)"""
+    Ho, Wo = (H + 2 * pad - dil * (k - 1) - 1) // stride + 1, (W + 2 * pad - dil * (k - 1) - 1) // stride + 1
+    g = torch.Generator().manual_seed(B + H + C + k)
+    x, w, b = torch.randn((B, H, W, C), generator=g), torch.randn((C, k * k), generator=g), torch.randn(C, generator=g)
+    R = torch.randn((B, Ho, Wo, C), generator=g)
+    xp = torch.zeros((B, H + 2 * pad, W + 2 * pad, C), dtype=torch.float64)
+    xp[:, pad:pad + H, pad:pad + W] = x
+    want, mag = b.double().expand(B, Ho, Wo, C).clone(), b.abs().double().expand(B, Ho, Wo, C).clone()
+    for t in range(k * k):
+        ky, kx = t // k * dil, t % k * dil
+        part = xp[:, ky:ky + (Ho - 1) * stride + 1:stride, kx:kx + (Wo - 1) * stride + 1:stride] * w[:, t].double()
+        want, mag = want + part, mag + part.abs()
+    if act == 0:
+        want = torch.relu(want)
+    elif act == 1:
+        want = 0.5 * want * (1 + torch.erf(want / 2 ** 0.5))
+    if res:
+        want = want + R.double()
+    geom = hipabi.ConvGeom(B, H, W, C, Ho, Wo, C, k, k, stride, stride, dil, dil, pad, pad, C)
+    dx, dw, db, y = x.cuda(), (w if transposed else w.t().contiguous()).cuda(), b.cuda(), R.cuda()
+    if res:
+        rc = L.knx_hip_conv_t_res(ctypes.byref(geom), ptr(dx), ptr(dw), ptr(db), act, 0.0, ptr(y), ptr(y), hipabi.stream())
+    else:
+        entry = L.knx_hip_conv_t if transposed else L.knx_hip_conv
+        rc = entry(ctypes.byref(geom), ptr(dx), ptr(dw), ptr(db), act, 0.0, ptr(y), hipabi.stream())
+    hipabi.check(rc)
+    lim = (k * k + 4) * 2.0 ** -24 * (mag + R.abs().double()) + (1e-6 * mag if act == 1 else 0)
+    assert torch.all((y.cpu().double() - want).abs() <= lim)
