@@ -56,8 +56,9 @@ __global__ void __launch_bounds__(256) softmax_kernel(const float* __restrict__ 
 }
 
 // ---- register-resident row kernels ----
-// G lanes per row (16, 32 or 64), NV float4 per lane: used when cols % 4 == 0, cols ≤ 4·G·NV and the rows are 16-byte
-// aligned.  Each row is read from memory once (16-byte loads) and kept in registers for every pass over it.
+// G lanes per row (16, 32 or 64), NV float4 per lane, cols ≤ 4·G·NV.  ODD: cols no multiple of 4 or rows not 16-byte aligned:
+// the same accesses at float alignment, a row's last values one by one (65,536 × 1001 softmax and layer_norm: three passes
+// of 4-byte accesses before).  Each row is read from memory once (16-byte loads) and kept in registers for every pass over it.
 template <int G>
 __device__ __forceinline__ float group_sum(float v)
 {
@@ -72,20 +73,54 @@ __device__ __forceinline__ float group_max(float v)
 }
 __device__ __forceinline__ float f4(const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
 
+typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte access at any float address
+
+// values 4q … 4q + 3 of a row of cols (past its end: fill), and back
+template <bool ODD>
+__device__ __forceinline__ float4 row_get(const float* p, int q, int cols, float fill)
+{
+    if (!ODD) return reinterpret_cast<const float4*>(p)[q];
+    if (4 * q + 3 < cols) {
+        const v4fu v = *reinterpret_cast<const v4fu*>(p + 4 * q);
+        return make_float4(v.x, v.y, v.z, v.w);
+    }
+    float4 v = make_float4(fill, fill, fill, fill);
+    if (4 * q + 0 < cols) v.x = p[4 * q + 0];
+    if (4 * q + 1 < cols) v.y = p[4 * q + 1];
+    if (4 * q + 2 < cols) v.z = p[4 * q + 2];
+    return v;
+}
+template <bool ODD>
+__device__ __forceinline__ void row_put(float* p, int q, int cols, const float4& v)
+{
+    if (!ODD) {
+        reinterpret_cast<float4*>(p)[q] = v;
+        return;
+    }
+    if (4 * q + 3 < cols) {
+        const v4fu u = {v.x, v.y, v.z, v.w};
+        *reinterpret_cast<v4fu*>(p + 4 * q) = u;
+        return;
+    }
+    if (4 * q + 0 < cols) p[4 * q + 0] = v.x;
+    if (4 * q + 1 < cols) p[4 * q + 1] = v.y;
+    if (4 * q + 2 < cols) p[4 * q + 2] = v.z;
+}
+
 // layer_norm of one row, same formulas as layernorm_kernel: lane l of the row's G lanes gets its float4 chunks
 // l, l + G, … of the normalized row in o (chunks past the row are left unset)
-template <int G, int NV>
+template <int G, int NV, bool ODD = false>
 __device__ __forceinline__ void ln_row(const float* x, int row, int cols, int l, const float* __restrict__ gamma,
                                        const float* __restrict__ beta, float eps, float4 (&o)[NV])
 {
-    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * cols);
-    const int nq = cols >> 2;
+    const float* xr = x + (size_t)row * cols;
+    const int nq = ODD ? (cols + 3) >> 2 : cols >> 2;
     float4 v[NV];
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int q = i * G + l;
-        v[i] = q < nq ? xr[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[i] = q < nq ? row_get<ODD>(xr, q, cols, 0.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
         s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
     const float mean = group_sum<G>(s) / (float)cols;
@@ -94,16 +129,18 @@ __device__ __forceinline__ void ln_row(const float* x, int row, int cols, int l,
     for (int i = 0; i < NV; ++i)
         if (i * G + l < nq)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { const float d = f4(v[i], e) - mean; ss += d * d; }
+            for (int e = 0; e < 4; ++e) {
+                const float d = f4(v[i], e) - mean;
+                if (!ODD || 4 * (i * G + l) + e < cols) ss += d * d;
+            }
     const float rstd = 1.0f / sqrtf(group_sum<G>(ss) / (float)cols + eps);
-    const float4* g4 = reinterpret_cast<const float4*>(gamma);  // 16-byte aligned (checked by the caller)
-    const float4* b4 = reinterpret_cast<const float4*>(beta);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int q = i * G + l;
         if (q >= nq) continue;
-        const float4 gq = gamma ? g4[q] : make_float4(1.f, 1.f, 1.f, 1.f);
-        const float4 bq = beta ? b4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        // (16-byte aligned unless ODD: checked by the caller)
+        const float4 gq = gamma ? row_get<ODD>(gamma, q, cols, 1.0f) : make_float4(1.f, 1.f, 1.f, 1.f);
+        const float4 bq = beta ? row_get<ODD>(beta, q, cols, 0.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
         float t4[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -118,7 +155,7 @@ __device__ __forceinline__ void ln_row(const float* x, int row, int cols, int l,
 }
 
 // layer_norm (x may alias y: every lane reads its whole row before writing)
-template <int G, int NV>
+template <int G, int NV, bool ODD>
 __global__ void __launch_bounds__(256) layernorm_vec(const float* x, float* y, int rows, int cols,
                                                       const float* __restrict__ gamma, const float* __restrict__ beta,
                                                       float eps)
@@ -126,12 +163,11 @@ __global__ void __launch_bounds__(256) layernorm_vec(const float* x, float* y, i
     const int row = blockIdx.x * (256 / G) + (int)threadIdx.x / G, l = threadIdx.x % G;
     if (row >= rows) return;
     float4 o[NV];
-    ln_row<G, NV>(x, row, cols, l, gamma, beta, eps, o);
-    float4* yr = reinterpret_cast<float4*>(y + (size_t)row * cols);
-    const int nq = cols >> 2;
+    ln_row<G, NV, ODD>(x, row, cols, l, gamma, beta, eps, o);
+    const int nq = ODD ? (cols + 3) >> 2 : cols >> 2;
 #pragma unroll
     for (int i = 0; i < NV; ++i)
-        if (i * G + l < nq) yr[i * G + l] = o[i];
+        if (i * G + l < nq) row_put<ODD>(y + (size_t)row * cols, i * G + l, cols, o[i]);
 }
 
 // layer_norm followed by the per-row int8 quantization of kernix_qmatmul (the steps of knx_hip_quantize_rows: s = m/127
@@ -184,19 +220,19 @@ __global__ void __launch_bounds__(256) layernorm_quant_vec(const float* x, int r
 }
 
 // softmax, same formulas as softmax_kernel; exp(x − max) is computed once and kept
-template <int G, int NV>
+template <int G, int NV, bool ODD>
 __global__ void __launch_bounds__(256) softmax_vec(const float* x, float* y, int rows, int cols)
 {
     const int row = blockIdx.x * (256 / G) + (int)threadIdx.x / G, l = threadIdx.x % G;
     if (row >= rows) return;
-    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * cols);
-    const int nq = cols >> 2;
+    const float* xr = x + (size_t)row * cols;
+    const int nq = ODD ? (cols + 3) >> 2 : cols >> 2;
     float4 v[NV];
     float m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int q = i * G + l;
-        v[i] = q < nq ? xr[q] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        v[i] = q < nq ? row_get<ODD>(xr, q, cols, -INFINITY) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
 #pragma unroll
         for (int e = 0; e < 4; ++e) m = f4(v[i], e) > m ? f4(v[i], e) : m;
     }
@@ -206,17 +242,18 @@ __global__ void __launch_bounds__(256) softmax_vec(const float* x, float* y, int
     for (int i = 0; i < NV; ++i) {
         if (i * G + l >= nq) continue;
         v[i] = make_float4(expf(v[i].x - m), expf(v[i].y - m), expf(v[i].z - m), expf(v[i].w - m));
+        const int left = ODD ? cols - 4 * (i * G + l) : 4;  // values of this quad inside the row
         s += v[i].x;
-        s += v[i].y;
-        s += v[i].z;
-        s += v[i].w;
+        if (left > 1) s += v[i].y;
+        if (left > 2) s += v[i].z;
+        if (left > 3) s += v[i].w;
     }
     const float inv = 1.0f / group_sum<G>(s);
-    float4* yr = reinterpret_cast<float4*>(y + (size_t)row * cols);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int q = i * G + l;
-        if (q < nq) yr[q] = make_float4(v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv);
+        if (q < nq)
+            row_put<ODD>(y + (size_t)row * cols, q, cols, make_float4(v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv));
     }
 }
 
@@ -230,6 +267,24 @@ __global__ void __launch_bounds__(256) softmax_vec(const float* x, float* y, int
         else if ((nq) <= 128) hipLaunchKernelGGL((K<64, 2>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
         else if ((nq) <= 256) hipLaunchKernelGGL((K<64, 4>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
         else hipLaunchKernelGGL((K<64, 8>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__);                \
+    } while (0)
+
+// the same for rows of any width up to 4096 (nq ≤ 1024) and alignment: K<G, NV, ODD>
+#define KNX_ROWVEC_ANY(K, odd, nq, rows, stream, ...)                                                      \
+    do {                                                                                                  \
+        if (odd) KNX_ROWVEC_ONE(K, true, nq, rows, stream, __VA_ARGS__);                                  \
+        else KNX_ROWVEC_ONE(K, false, nq, rows, stream, __VA_ARGS__);                                     \
+    } while (0)
+#define KNX_ROWVEC_ONE(K, O, nq, rows, stream, ...)                                                                    \
+    do {                                                                                                              \
+        hipStream_t st_ = knx::as_stream(stream);                                                                     \
+        if ((nq) <= 16) hipLaunchKernelGGL((K<16, 1, O>), dim3(((rows) + 15) / 16), dim3(256), 0, st_, __VA_ARGS__);  \
+        else if ((nq) <= 32) hipLaunchKernelGGL((K<32, 1, O>), dim3(((rows) + 7) / 8), dim3(256), 0, st_, __VA_ARGS__); \
+        else if ((nq) <= 64) hipLaunchKernelGGL((K<64, 1, O>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
+        else if ((nq) <= 128) hipLaunchKernelGGL((K<64, 2, O>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
+        else if ((nq) <= 256) hipLaunchKernelGGL((K<64, 4, O>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
+        else if ((nq) <= 512) hipLaunchKernelGGL((K<64, 8, O>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__); \
+        else hipLaunchKernelGGL((K<64, 16, O>), dim3(((rows) + 3) / 4), dim3(256), 0, st_, __VA_ARGS__);              \
     } while (0)
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -504,8 +559,9 @@ extern "C" int knx_hip_layernorm(const float* x, float* y, int rows, int cols, c
     KNX_REQUIRE(rows >= 0 && cols >= 1, name);
     if (rows == 0) return KNX_OK;
     KNX_REQUIRE(x && y, name);
-    if (cols % 4 == 0 && cols / 4 <= 512 && aligned16(x) && aligned16(y) && aligned16(gamma) && aligned16(beta)) {
-        KNX_ROWVEC_DISPATCH(layernorm_vec, cols / 4, rows, stream, x, y, rows, cols, gamma, beta, eps);
+    if (cols <= 4096) {
+        const bool odd = cols % 4 != 0 || !aligned16(x) || !aligned16(y) || !aligned16(gamma) || !aligned16(beta);
+        KNX_ROWVEC_ANY(layernorm_vec, odd, (cols + 3) / 4, rows, stream, x, y, rows, cols, gamma, beta, eps);
         return knx::check_launch(name);
     }
     KNX_LAUNCH(name, layernorm_kernel, (rows + 3) / 4, x, y, rows, cols, gamma, beta, eps);
@@ -530,8 +586,9 @@ extern "C" int knx_hip_softmax(const float* x, float* y, int rows, int cols, voi
     KNX_REQUIRE(rows >= 0 && cols >= 1, name);
     if (rows == 0) return KNX_OK;
     KNX_REQUIRE(x && y, name);
-    if (cols % 4 == 0 && cols / 4 <= 512 && aligned16(x) && aligned16(y)) {
-        KNX_ROWVEC_DISPATCH(softmax_vec, cols / 4, rows, stream, x, y, rows, cols);
+    if (cols <= 4096) {
+        const bool odd = cols % 4 != 0 || !aligned16(x) || !aligned16(y);
+        KNX_ROWVEC_ANY(softmax_vec, odd, (cols + 3) / 4, rows, stream, x, y, rows, cols);
         return knx::check_launch(name);
     }
     KNX_LAUNCH(name, softmax_kernel, (rows + 3) / 4, x, y, rows, cols);

@@ -1,5 +1,5 @@
 """fp32 products on the bf16 matrix cores (knx_xgemm.hip): every tile at its edges, odd strides and addresses, values
-that have no finite bf16 parts."""
+that have no finite bf16 parts; depthwise convolutions; rows of any width and alignment."""
 import ctypes
 
 import numpy as np
@@ -165,3 +165,37 @@ def test_depthwise(L, B, H, W, C, k, stride, dil, pad, transposed, act, res):
     hipabi.check(rc)
     lim = (k * k + 4) * 2.0 ** -24 * (mag + R.abs().double()) + (1e-6 * mag if act == 1 else 0)
     assert torch.all((y.cpu().double() - want).abs() <= lim)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 2), (5, 63), (17, 65), (9, 127), (4, 130), (6, 257), (3, 513), (2, 1001), (2, 2047),
+                                       (3, 2051), (2, 4094), (2, 4095), (2, 4096), (2, 4097)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rows_of_any_width(L, rows, cols, offset):
+    """layer_norm and softmax at every lanes-per-row choice, with a ragged last quad or a row address that is no multiple of
+    16 bytes; masked entries and a masked row as the definition has them; nothing past a row is written.  Sums of n values
+    in fp32 trees and chains of at most 64 per lane: 70 roundings and the exponential's."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x, ga, be = torch.randn((rows, cols), generator=g) * 2, 1 + torch.randn(cols, generator=g) * 0.05, torch.randn(cols, generator=g)
+    buf = torch.zeros(rows * cols + offset + 1)
+    buf[offset:offset + rows * cols] = x.flatten()
+    dx, y = buf.cuda(), torch.full((rows * cols + offset + 1,), 7.0, device="cuda")
+    dg, db = ga.cuda(), be.cuda()
+    at = lambda t: ctypes.c_void_p(t.data_ptr() + 4 * offset)  # noqa: E731
+    hipabi.check(L.knx_hip_layernorm(at(dx), at(y), rows, cols, ptr(dg), ptr(db), 1e-5, hipabi.stream()))
+    got = y.cpu()
+    assert got[-1] == 7.0 and torch.all(got[:offset] == 7.0)
+    xd = x.double()
+    m = xd.mean(1, keepdim=True)
+    sd = torch.sqrt(((xd - m) ** 2).mean(1, keepdim=True) + 1e-5)
+    want = (xd - m) / sd * ga.double() + be.double()
+    lim = 70 * 2.0 ** -24 * ((xd.abs() + m.abs() + xd.abs().mean(1, keepdim=True)) / sd * ga.abs().double() * 2 + be.abs().double())
+    assert torch.all((got[offset:-1].double().reshape(rows, cols) - want).abs() <= lim)
+    if cols > 2:
+        x[0, 1], x[-1, cols - 1] = -float("inf"), -float("inf")
+        buf[offset:offset + rows * cols] = x.flatten()
+        dx = buf.cuda()
+    hipabi.check(L.knx_hip_softmax(at(dx), at(y), rows, cols, hipabi.stream()))
+    got = y.cpu()
+    assert got[-1] == 7.0 and torch.all(got[:offset] == 7.0)
+    want = torch.softmax(x.double(), 1)
+    assert torch.all((got[offset:-1].double().reshape(rows, cols) - want).abs() <= (70 + 24) * 2.0 ** -24 * want)
