@@ -197,7 +197,7 @@ typedef struct {
 KNX_API int knx_hip_conv(const knx_conv_geom* g, const float* x, const float* w, const float* bias, int act,
                          float alpha, float* y, void* stream);
 /* Same with the weight transposed: Wt Co × (kh·kw·C/groups), the device layout of the model's convolution weights.
- * Channel counts per group that are multiples of 32 run on the pipelined implicit GEMM (LDS-DMA gathers). */
+ * At most 64 taps and kh·kw·C/groups ≥ 16: the implicit GEMM on the bf16 matrix cores, at fp32 accuracy. */
 KNX_API int knx_hip_conv_t(const knx_conv_geom* g, const float* x, const float* wt, const float* bias, int act,
                            float alpha, float* y, void* stream);
 /* y = act(conv(x, Wt) + bias) + R (R the same shape as y; R may equal y): a CONV followed by the BINARY add of R

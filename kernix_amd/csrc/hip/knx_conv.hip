@@ -1,4 +1,6 @@
-// knx_conv.hip — NHWC convolution as an implicit GEMM on v_mfma_f32_32x32x2_f32 (gfx950).
+// knx_conv.hip — NHWC convolution (gfx950): the dispatch, the first layers' kernel, depthwise convolutions and the general
+// implicit GEMM on v_mfma_f32_32x32x2_f32.  Weights stored transposed (Co × K, the model's) with K ≥ 16 and at most 64 taps run
+// on the bf16 matrix cores instead (knx_xconv, knx_xgemm.hip).
 //
 // Replaces kernix_conv_run's tiled im2col → cblas_sgemm → bias_act (reference include/kernix_model.h:711-771,
 // im2col :677-693): the GEMM is out[m][n] = Σ_k A[m][k]·W[k][n] with m = (b, oy, ox), k = (ky, kx, ci) and
