@@ -569,7 +569,7 @@ int conv_entry(const knx_conv_geom* g, const float* x, const float* w, const flo
         // KNX_CONV_TILE forces a tile of the bf16 kernel (tests, tuning)
         static const struct { const char* name; int tile; } TILES[] = {
             {"256x256", KNX_X256x128}, {"256x128", KNX_X256x128}, {"128x128", KNX_X128x128}, {"128x128w8", KNX_X128x128},
-            {"64x128", KNX_X64x64}, {"256x64", KNX_X256x64}, {"128x64", KNX_X128x64}};
+            {"64x128", KNX_X64x64}, {"256x64", KNX_X256x64}, {"128x64", KNX_X128x64}, {"64x64k2", KNX_X64x64K2}};
         const char* force = getenv("KNX_CONV_TILE");
         int tile = 0;
         for (const auto& t : TILES)

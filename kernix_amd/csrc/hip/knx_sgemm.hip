@@ -569,7 +569,7 @@ int dispatch_nt(SgArgs p, int batch, hipStream_t s, const char* name)
     const char* force = getenv("KNX_SGEMM_KERNEL");
     if (force != nullptr && *force) {
         static const struct { const char* name; int tile; } TILES[] = {
-            {"t256", KNX_X256x256}, {"t128", KNX_X256x128}, {"t128w8", KNX_X128x128}, {"t64", KNX_X128x64}, {"t64x64", KNX_X64x64}};
+            {"t256", KNX_X256x256}, {"t128", KNX_X256x128}, {"t128w8", KNX_X128x128}, {"t64", KNX_X128x64}, {"t64x64", KNX_X64x64}, {"t64x64k2", KNX_X64x64K2}};
         for (const auto& t : TILES)
             if (strcmp(force, t.name) == 0) {
                 const int rc = knx_xgemm(p, batch, t.tile, s, name);

@@ -75,8 +75,11 @@ __device__ __forceinline__ const float* tap_at(const window& w, int2 e)
 // where a plain bf16 GEMM of torch's reaches 1150 on the same card; fp32 instructions: 147 TFLOP/s); the smaller tiles
 // the split's instructions and the LDS, which overlap the multiplies only in part (128×128: 54% of the matrix cores'
 // cycles).  K-tiles of 32 or 64 values per barrier, four k-tiles of loads in flight and four waves of 64×64 were slower.
-template <int BM, int BN, int WM, int WN, int OCC, bool PIPE, int MODE>
-__global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
+// KG = 2: two groups of WM×WN waves, each with stages of its own, take alternate k-tiles of the same outputs, and the second
+// hands its sums to the first through LDS at the end: for shapes that give a CU one workgroup, whose waves would wait for
+// one another's LDS reads and splits alone.
+template <int BM, int BN, int WM, int WN, int OCC, bool PIPE, int MODE, int KG>
+__global__ void __launch_bounds__(WM * WN * 64 * KG, OCC) xgemm(knx_xargs p)
 {
     constexpr int NW = WM * WN, NT = NW * 64;
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
@@ -84,11 +87,15 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     constexpr int STAGE = (BM + BN) / 32 * 3 * 1024;
     constexpr int P = (BM + BN) * Q / NT, PA = BM * Q / NT;  // pieces per thread and k-tile; of A
     static_assert(BM * Q % NT == 0 && BN * Q % NT == 0 && TM % 32 == 0 && TN % 32 == 0, "load split");
-    __shared__ __attribute__((aligned(16))) int8_t lds0[STAGE];
-    __shared__ __attribute__((aligned(16))) int8_t lds1[STAGE];
+    static_assert(KG == 1 || (KG == 2 && PIPE), "groups of waves");
+    __shared__ __attribute__((aligned(16))) int8_t lds0s[KG * STAGE];
+    __shared__ __attribute__((aligned(16))) int8_t lds1s[KG * STAGE];
 
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lane = threadIdx.x & 63;
+    const int all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int kg = KG == 1 ? 0 : all / NW, wave = KG == 1 ? all : all % NW, t = wave * 64 + lane;  // of this wave's group
+    int8_t* const lds0 = lds0s + kg * STAGE;
+    int8_t* const lds1 = lds1s + kg * STAGE;
     const int wm = wave / WN, wn = wave % WN;
     int tm, tn;
     tile_of_best(blockIdx.x, p.tiles_m, p.tiles_n, BM, BN, tm, tn);
@@ -112,7 +119,7 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     extern __shared__ __attribute__((aligned(16))) int2 taps[];
     const int cbase = MODE == PLAIN ? 0 : (int)blockIdx.y * p.cgc;
     if (MODE != PLAIN) {
-        for (int i = t; i < (MODE == CONV4 ? K / 4 : K); i += NT) {
+        for (int i = threadIdx.x; i < (MODE == CONV4 ? K / 4 : K); i += NT * KG) {
             const int k = MODE == CONV4 ? 4 * i : i, tap = k / p.cgc, ky = tap / p.cv.kw, kx = tap - ky * p.cv.kw;
             taps[i] = make_int2((int)((((long long)ky * p.cv.dh * p.cv.W + (long long)kx * p.cv.dw) * p.cv.C + (k - tap * p.cgc)) * 4), tap);
         }
@@ -158,8 +165,14 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
         return v;
     };
     const int part = K % KT, nkt = (K + KT - 1) / KT, shift = part ? KT - part : 0;
+    // (KG = 2: this group's k-tile kt is tile 2·kt + kg; past the last one, which the other group may still have, zeros)
     auto gload = [&](int kt, float4 (&v)[P]) __attribute__((always_inline)) {
-        const int k = min(kt, nkt - 1) * KT - shift;
+        const int tile = kt * KG + kg, k = min(tile, nkt - 1) * KT - shift;
+        if (KG > 1 && tile >= nkt) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < P; ++i) {
             if (MODE != PLAIN && i < PA) v[i] = gather4(win[i], k + 4 * q);
@@ -168,7 +181,7 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
         }
     };
     auto gload_first = [&](float4 (&v)[P]) __attribute__((always_inline)) {
-        if (part == 0) return gload(0, v);
+        if (part == 0 || kg > 0) return gload(0, v);
 #pragma unroll
         for (int i = 0; i < P; ++i) {
             if (MODE != PLAIN && i < PA) v[i] = gather4_tail(win[i], 4 * q, part - 4 * q);
@@ -283,13 +296,14 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
             gload(kt + j + 2 + D, v[(j + 2) % D]);
             handover();
         };
+        const int steps = (nkt + KG - 1) / KG;
         int kt = 0;
-        for (; kt + D <= nkt; kt += D)
+        for (; kt + D <= steps; kt += D)
 #pragma unroll
             for (int j = 0; j < D; ++j) step(kt, j);
 #pragma unroll
         for (int j = 0; j < D - 1; ++j)
-            if (kt + j < nkt) step(kt, j);
+            if (kt + j < steps) step(kt, j);
     } else {
         float4 w0[P];
         gload_first(w0);
@@ -319,6 +333,25 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[0][0][e] = acc[0][0][e] + accs[NA - 1][0][0][e];
 
+    if (KG == 2) {  // the second group's sums to the first (every wave is past its last read of the stages)
+        float* part_sums = reinterpret_cast<float*>(lds0s) + wave * FM * FN * 1024 + lane;
+        static_assert(KG == 1 || NW * FM * FN * 4096 <= KG * STAGE, "the sums fit the first stages");
+        if (kg == 1)
+#pragma unroll
+            for (int fi = 0; fi < FM; ++fi)
+#pragma unroll
+                for (int fj = 0; fj < FN; ++fj)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) part_sums[((fi * FN + fj) * 16 + e) * 64] = acc[fi][fj][e];
+        handover();
+        if (kg == 1) return;
+#pragma unroll
+        for (int fi = 0; fi < FM; ++fi)
+#pragma unroll
+            for (int fj = 0; fj < FN; ++fj)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[fi][fj][e] = acc[fi][fj][e] + part_sums[((fi * FN + fj) * 16 + e) * 64];
+    }
     // a non-finite accumulator: this wave's outputs again, in fp32 products
     float nan = 0.0f;
 #pragma unroll
@@ -440,14 +473,14 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) xgemm(knx_xargs p)
     }
 }
 
-template <int MODE, int BM, int BN, int WM, int WN, int OCC, bool PIPE>
+template <int MODE, int BM, int BN, int WM, int WN, int OCC, bool PIPE, int KG = 1>
 int launch(knx_xargs p, int batch, hipStream_t s, const char* name)
 {
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     const unsigned taps = MODE == PLAIN ? 0 : (unsigned)(MODE == CONV4 ? p.K / 4 : p.K) * 8;
-    hipLaunchKernelGGL((xgemm<BM, BN, WM, WN, OCC, PIPE, MODE>), dim3((unsigned)p.tiles_m * (unsigned)p.tiles_n, batch),
-                       dim3(WM * WN * 64), taps, s, p);
+    hipLaunchKernelGGL((xgemm<BM, BN, WM, WN, OCC, PIPE, MODE, KG>), dim3((unsigned)p.tiles_m * (unsigned)p.tiles_n, batch),
+                       dim3(WM * WN * 64 * KG), taps, s, p);
     return knx::check_launch(name);
 }
 
@@ -459,6 +492,7 @@ int launch_tile(const knx_xargs& p, int batch, int tile, hipStream_t s, const ch
     case KNX_X256x128: return launch<MODE, 256, 128, 4, 2, 1, true>(p, batch, s, name);
     case KNX_X256x64: return launch<MODE, 256, 64, 4, 1, 2, true>(p, batch, s, name);
     case KNX_X128x128: return launch<MODE, 128, 128, 4, 2, 1, true>(p, batch, s, name);
+    case KNX_X64x64K2: return launch<MODE, 64, 64, 2, 2, 1, true, 2>(p, batch, s, name);
     case KNX_X128x64: return launch<MODE, 128, 64, 2, 2, 2, true>(p, batch, s, name);
     default: return launch<MODE, 64, 64, 2, 2, 2, true>(p, batch, s, name);
     }
@@ -466,8 +500,9 @@ int launch_tile(const knx_xargs& p, int batch, int tile, hipStream_t s, const ch
 
 // The tile for a shape: the one with the least estimated time, workgroups per CU in whole rounds.  Per tile: µs for 16
 // values of k where at most half of the CUs have a workgroup and where all are busy, and µs for the prologue and the
-// epilogue, from 500×1000×2000, 8192×512×{512, 2048} and 4096³ on every tile (the tiles picked here: 41, 28, 88 and
-// 581 µs; on v_mfma_f32_32x32x2_f32 they took 83, 40, 130 and 930 µs).  Two choices the times make: 256×256 tiles, the
+// epilogue, from 500×1000×2000, 8192×512×{512, 2048} and 4096³ on every tile (the tiles picked here: 37, 28, 88 and
+// 581 µs; on v_mfma_f32_32x32x2_f32 they took 83, 40, 130 and 930 µs).  Three choices the times make: two groups of waves on
+// a 64×64 tile where each CU has at most one (500×1000×2000: 36.5 against 41 µs, 74 images of 14×14×137 → 46: 34 against 49), 256×256 tiles, the
 // fewest operand bytes per multiply, wherever they come in full rounds and K is long (4096³: 581 µs, against 602 on
 // 256×128 and 652 on 128×128); 64×64 where larger tiles would leave CUs idle.
 int pick_tile(const knx_xargs& p, int batch, bool conv, float* us)
@@ -480,6 +515,7 @@ int pick_tile(const knx_xargs& p, int batch, bool conv, float* us)
              {KNX_X256x64, 256, 64, 0.78f, 0.65f, 9.0f, 4.0f},
              {KNX_X128x128, 128, 128, 0.41f, 0.63f, 8.0f, 2.0f},
              {KNX_X128x64, 128, 64, 0.37f, 0.37f, 7.5f, 5.0f},
+             {KNX_X64x64K2, 64, 64, 0.23f, 0.24f, 7.5f, 1.5f},
              {KNX_X64x64, 64, 64, 0.26f, 0.21f, 7.0f, 1.5f}};
     int best = KNX_X64x64;
     *us = 0.0f;

@@ -62,7 +62,7 @@ struct knx_xargs {
 };
 
 // the output tile of a workgroup; 0: picked by the shape
-enum { KNX_X64x64 = 1, KNX_X128x64, KNX_X256x64, KNX_X128x128, KNX_X256x128, KNX_X256x256 };
+enum { KNX_X64x64 = 1, KNX_X64x64K2, KNX_X128x64, KNX_X256x64, KNX_X128x128, KNX_X256x128, KNX_X256x256 };
 
 // Both return 1 without launching where the shape does not fit (the caller has a general kernel).
 int knx_xgemm(const knx_xargs& p, int batch, int tile, hipStream_t s, const char* name);

@@ -12,7 +12,7 @@ from kernix_amd.hipabi import ptr  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
-TILES = ["t256", "t128", "t128w8", "t64", "t64x64"]
+TILES = ["t256", "t128", "t128w8", "t64", "t64x64", "t64x64k2"]
 
 
 @pytest.fixture(scope="module")
@@ -102,7 +102,7 @@ def test_values_without_finite_parts(L, tile, monkeypatch):
 
 @pytest.mark.parametrize("C,Co,k,stride,dil,groups", [(24, 80, 3, 2, 1, 1), (7, 20, 5, 1, 1, 1), (91, 62, 1, 1, 1, 1),
                                                       (64, 130, 3, 1, 2, 1), (36, 24, 3, 1, 1, 2), (30, 22, 3, 1, 1, 2)])
-@pytest.mark.parametrize("tile", ["256x128", "256x64", "128x128", "128x64", "64x128"])
+@pytest.mark.parametrize("tile", ["256x128", "256x64", "128x128", "128x64", "64x128", "64x64k2"])
 def test_convolution(L, C, Co, k, stride, dil, groups, tile, monkeypatch):
     """channel counts that are multiples of 4 and that are not, an infinite and a NaN pixel; against a direct sum"""
     monkeypatch.setenv("KNX_CONV_TILE", tile)
